@@ -727,6 +727,11 @@ struct MfmaLayer {
     //      c = 16 t + 4 (n >> 2) + i, f = 16 + 2 (n & 3) + fb for row group q; after them the lane
     //      holds c = 16 t + cb + 2 h and f = 16 + 2 (n & 3) + (q >> 1).  f = D0 is the bias; the sum of g
     //      over the wave's rows (db2) has gathered in the first padded hidden unit ----
+    // (The swaps read the accumulators from inside assembly statements, where the compiler does not count the wait
+    // states a vector instruction needs after a matrix instruction wrote its operand: up to 11, covered here.)
+    asm volatile("s_nop 15"
+                 : "+v"(dacc_f[0][0]), "+v"(dacc_f[0][1]), "+v"(dacc_f[1][0]), "+v"(dacc_f[1][1]), "+v"(dacc_f[2][0]),
+                   "+v"(dacc_f[2][1]));
     const int cb = 4 * (n >> 2) + (q & 1);
     const int f = 16 + 2 * (n & 3) + (q >> 1);
 #pragma unroll

@@ -563,10 +563,11 @@ struct MfmaSplitLayer {
   template <int LIK>
   __device__ __forceinline__ void write_partials(float* slot, const float*, bool last) {
     const int lane = opaque_tid() & 63, n = lane & 15, q = lane >> 4, c8 = n & 7;
-    // The lane swaps below read the accumulators from inside assembly statements, where the compiler does not
-    // count the wait states a vector instruction needs after a matrix instruction wrote its operand (up to 11).
-    // Once per step: sixteen wait states here cover whatever the tile loop ended on.
-    asm volatile("s_nop 15" ::: "memory");
+    // The lane swaps below read this accumulator from inside assembly statements, where the compiler does not count
+    // the wait states a vector instruction needs after a matrix instruction wrote its operand (up to 11).  Once per
+    // step: sixteen wait states here cover whatever the tile loop ended on; the accumulator is an operand, so that no
+    // swap can be scheduled before them.
+    asm volatile("s_nop 15" : "+v"(dacc_e[NT]));
     // ---- hidden 0 .. 31: lane (n, q), component i: c = 16 t + 4 q + i, f = n and f = 16 + c8 (lanes n and n ^ 8
     //      store the same bits to the same place) ----
 #pragma unroll
