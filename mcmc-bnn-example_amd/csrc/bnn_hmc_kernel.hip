@@ -295,6 +295,7 @@ __global__ __launch_bounds__(T) void hmc_kernel(const KArgs a) {
   cx.wave = wave;
   cx.partner = wave ^ (W / 2);
   cx.tile_lds = s_tile[wave];
+  cx.w_lds = s_w;
 
   const ModelConsts mc = a.mc;
   // records of flagged packets (8 bytes per parameter), two per workgroup (by step parity)
@@ -816,6 +817,7 @@ __global__ __launch_bounds__(512) void loss_kernel(const LossArgs a) {
     cx.tile_end = (int)((long)a.n_tiles * (gw + 1) / GW);
   }
   cx.tile_lds = s_tile[wave];
+  cx.w_lds = s_w;
   __syncthreads();
   Layer layer;
   layer.prime(cx);

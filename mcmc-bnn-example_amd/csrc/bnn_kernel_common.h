@@ -124,6 +124,22 @@ __device__ __forceinline__ float lane_fold16(float a, float b) {
   return a + b;
 }
 
+// D = A B + C on v_mfma_f32_16x16x4_f32: lane 16 q + n holds A[n][q], B[q][n] and C[4 q + j][n] (j < 4)
+__device__ __forceinline__ f4 mfma_f32(float a, float b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Whether a wave has to take its tiles again, those with a NaN among their row sums in FP32: a lane's sum over rows is
+// NaN (`nan_sum`) because a feature or a weight has no bf16 parts -- or is a NaN itself.  With a NaN among the weights every row is
+// NaN in any arithmetic: so it is from some step on in a diverged trajectory, whose steps must not take longer than others.
+// The same answer in every lane.
+__device__ __forceinline__ bool again_in_fp32(bool nan_sum, const float* weights, int count) {
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan_sum) == 0, 1)) return false;
+  bool nan = false;
+  for (int i = opaque_tid() & 63; i < count; i += 64) nan |= __builtin_isnan(weights[i]);
+  return __builtin_amdgcn_ballot_w64(nan) == 0;
+}
+
 // sum over the 8 lanes of a half row
 __device__ __forceinline__ float row8_allreduce(float v) {
   v += dpp_move<0xB1>(v);
@@ -285,6 +301,7 @@ struct StepCtx {
   int* progress;          // LDS, one word per wave: tiles done in this step (null = no balancing)
   int wave, partner;      // this wave and the wave it shares a SIMD with
   float* tile_lds;        // LDS, this wave's copy of the tile it is working on (layers that keep one)
+  const float* w_lds;     // LDS, the weights of this step
   int back, back_next;    // this gradient evaluation / the next one walks a wave's tiles backwards (layers that
                           // alternate; see leapfrog_walks_back)
 };

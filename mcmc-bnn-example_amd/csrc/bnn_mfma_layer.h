@@ -637,11 +637,11 @@ struct MfmaLayer {
       issue(C);
       wait_tile<2 * N_LOADS>(A);
       compute(A, i);
-    }
-    if (left == 2) {
-      issue(A);
-      wait_tile<2 * N_LOADS>(B);
-      compute(B, i + 1);
+      if (left == 2) {
+        issue(A);
+        wait_tile<2 * N_LOADS>(B);
+        compute(B, i + 1);
+      }
     }
     // no register of a set may be used or reused before its last load has landed
     wait_tile<0>(A);

@@ -161,9 +161,30 @@ struct MfmaSplitLayer {
     return __builtin_bit_cast(bf4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p));
   }
 
+  // GEMM1 of a tile in FP32: x_aug, read again from memory (rows past the end: the last row), times W1_aug from the
+  // FP32 weights in LDS, scaled afterwards (k times a large finite weight may be infinite).  The result as GEMM1 leaves
+  // it, hidden 32 .. 39 in both column halves.
+  __device__ __forceinline__ void gemm1_fp32(const StepCtx& cx, int row0, int n, int q, f4 (&acc)[NT], f4& acc5) const {
+    const float* row = cx.X + (size_t)min(row0 + n, cx.n - 1) * D0;
+    acc[0] = acc[1] = acc5 = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int i = 0; i < KS; ++i) {
+      const int k = KS * q + i;
+      const float x = k < D0 ? row[min(k, D0 - 1)] : (k == D0 ? 1.0f : 0.0f);
+      const float* w = cx.w_lds + min(k, D0) * D1;
+      acc[0] = mfma_f32(x, k <= D0 ? w[n] : 0.0f, acc[0]);
+      acc[1] = mfma_f32(x, k <= D0 ? w[16 + n] : 0.0f, acc[1]);
+      acc5 = mfma_f32(x, k <= D0 ? w[32 + (n & 7)] : 0.0f, acc5);
+    }
+    acc[0] *= kExp2Scale;
+    acc[1] *= kExp2Scale;
+    acc5 *= kExp2Scale;
+  }
+
   // One tile: the LDS copy, GEMM1, the pointwise stage, GEMM2.  `tile` is this wave's LDS buffer.
-  // (GRAD == false: the forward half, for sums of the log-likelihood rows alone.)
-  template <int LIK, bool LAST, bool FULL, bool GRAD = true>
+  // (GRAD == false: the forward half, for sums of the log-likelihood rows alone.  FP32: where a row sum is NaN,
+  // GEMM1 in FP32.)
+  template <int LIK, bool LAST, bool FULL, bool GRAD = true, bool FP32 = false>
   __device__ __forceinline__ void compute_tile(const TileIn& ti, float* tile, const StepCtx& cx,
                                                const ModelConsts& mc, int row0, int n, int q) {
     const int r = n & 3, h8 = n >> 3;
@@ -172,15 +193,7 @@ struct MfmaSplitLayer {
 #pragma unroll
     for (int i = 0; i < KP; ++i) split2(ti.xa[i], xh[i], xm[i], xl[i]);
     __bf16* parts = reinterpret_cast<__bf16*>(tile);
-    if constexpr (GRAD) {
-      bf2* dst = reinterpret_cast<bf2*>(parts + n * 24 + KS * q);
-#pragma unroll
-      for (int i = 0; i < KP; ++i) {
-        dst[i] = xh[i];
-        dst[PART / 2 + i] = xm[i];
-        dst[2 * (PART / 2) + i] = xl[i];
-      }
-    }
+    if constexpr (GRAD) store_parts(parts, n, q, xh, xm, xl);
     const bf8 ah = operand(xh, pad_h), am = operand(xm, pad_m), al = operand(xl, pad_l);
     // ---- GEMM1, the small products first ----
     f4 acc[NT] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
@@ -205,7 +218,7 @@ struct MfmaSplitLayer {
     // (a part that several operands hold is read once for each: moving it would take vector instructions; the
     // second address is one the compiler does not know to be the first)
     bf8 be_lh, be_hm, be_mh, bf_hm, bf_lh;
-    if constexpr (GRAD) {
+    auto read_operands = [&] {
       const __bf16* rowp = parts + (4 * q + (n >> 2)) * 24;
       const __bf16* zeros = parts + 3 * PART;
       const __bf16* row2 = rowp + pad_h;
@@ -218,7 +231,8 @@ struct MfmaSplitLayer {
       const __bf16* f_hm = rowf + (r < 2 ? 0 : PART);
       bf_hm = join(read_transposed(f_hm), read_transposed(f_hm + pad_l));
       bf_lh = join(read_transposed(r < 2 ? rowf + 2 * PART : zeros), read_transposed(r < 2 ? rowf : zeros));
-    }
+    };
+    if constexpr (GRAD) read_operands();
     __builtin_amdgcn_sched_barrier(0);
     // ---- hidden 32 .. 39: the products of the two column halves; lanes n < 8 keep rows 4 q, 4 q + 1 (registers
     //      0, 1), lanes n >= 8 rows 4 q + 2, 4 q + 3 (registers 2, 3) ----
@@ -230,29 +244,48 @@ struct MfmaSplitLayer {
       sb = h8 == 0 ? t1 : t3;
     }
     // ---- pointwise stage (logistic form, see MfmaLayer::pointwise) ----
-    float yh[4] = {y_0, y_0, y_0, y_0};
+    float rz;
+    auto row_sums = [&] {
+      float yh[4] = {y_0, y_0, y_0, y_0};
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
+      for (int t = 0; t < NT; ++t) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float e = __builtin_amdgcn_exp2f(acc[t][j]);
-        const float sg = __builtin_amdgcn_rcpf(1.0f + e);
-        acc[t][j] = sg;
-        yh[j] = __builtin_fmaf(w2g[t], sg, yh[j]);
+        for (int j = 0; j < 4; ++j) {
+          const float e = __builtin_amdgcn_exp2f(acc[t][j]);
+          const float sg = __builtin_amdgcn_rcpf(1.0f + e);
+          acc[t][j] = sg;
+          yh[j] = __builtin_fmaf(w2g[t], sg, yh[j]);
+        }
+      }
+      sa = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sa));
+      sb = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sb));
+      // hidden 32 .. 39 in the row sums: a lane holds two of its four rows
+      asm("s_nop 1\n\t"
+          "v_fmac_f32_dpp %[y0], %[a], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0x3\n\t"
+          "v_fmac_f32_dpp %[y2], %[a], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xc\n\t"
+          "v_fmac_f32_dpp %[y1], %[b], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0x3\n\t"
+          "v_fmac_f32_dpp %[y3], %[b], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xc"
+          : [y0] "+v"(yh[0]), [y1] "+v"(yh[1]), [y2] "+v"(yh[2]), [y3] "+v"(yh[3])
+          : [a] "v"(sa), [b] "v"(sb), [w] "v"(w2g5));
+      // (y - yhat - b2) k2 of the four rows 4 q + j, in bank j of one register
+      rz = row16_reduce4(yh[0], yh[1], yh[2], yh[3]) + __builtin_fmaf(ti.y1, k2v, rho);
+    };
+    row_sums();
+    if constexpr (FP32) {
+      if (__builtin_amdgcn_ballot_w64(__builtin_isnan(rz)) != 0) {
+        gemm1_fp32(cx, row0, n, q, acc, acc5);
+        sa = h8 == 0 ? acc5[0] : acc5[2];
+        sb = h8 == 0 ? acc5[1] : acc5[3];
+        row_sums();
+        if constexpr (GRAD) {
+          // (a finite feature keeps finite parts in GEMM2; an infinite one makes NaN of its own weights' gradient)
+#pragma unroll
+          for (int i = 0; i < KP; ++i) split2_any(ti.xa[i], xh[i], xm[i], xl[i]);
+          store_parts(parts, n, q, xh, xm, xl);
+          read_operands();
+        }
       }
     }
-    sa = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sa));
-    sb = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sb));
-    // hidden 32 .. 39 in the row sums: a lane holds two of its four rows
-    asm("s_nop 1\n\t"
-        "v_fmac_f32_dpp %[y0], %[a], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0x3\n\t"
-        "v_fmac_f32_dpp %[y2], %[a], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xc\n\t"
-        "v_fmac_f32_dpp %[y1], %[b], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0x3\n\t"
-        "v_fmac_f32_dpp %[y3], %[b], %[w] quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xc"
-        : [y0] "+v"(yh[0]), [y1] "+v"(yh[1]), [y2] "+v"(yh[2]), [y3] "+v"(yh[3])
-        : [a] "v"(sa), [b] "v"(sb), [w] "v"(w2g5));
-    // (y - yhat - b2) k2 of the four rows 4 q + j, in bank j of one register
-    const float rz = row16_reduce4(yh[0], yh[1], yh[2], yh[3]) + __builtin_fmaf(ti.y1, k2v, rho);
     float gz = rz, dz = rz;
     if (LIK == 0) {
       dz = rz * ratio;
@@ -352,6 +385,17 @@ struct MfmaSplitLayer {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     return __builtin_bit_cast(bf8, u4{__builtin_bit_cast(unsigned, p[0]), __builtin_bit_cast(unsigned, p[1]),
                                       __builtin_bit_cast(unsigned, p[2]), zeros});
+  }
+  // lane (n, q)'s parts in the wave's copy of the tile
+  static __device__ __forceinline__ void store_parts(__bf16* parts, int n, int q, const bf2 (&h)[KP], const bf2 (&m)[KP],
+                                                     const bf2 (&l)[KP]) {
+    bf2* dst = reinterpret_cast<bf2*>(parts + n * 24 + KS * q);
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      dst[i] = h[i];
+      dst[PART / 2 + i] = m[i];
+      dst[2 * (PART / 2) + i] = l[i];
+    }
   }
   // two values in the slots of rows 0, 1 (lanes n < 8) or 2, 3 of the four, zeros in the others
   static __device__ __forceinline__ bf4 rows_of_half(bf2 v, int h8) {
@@ -501,11 +545,11 @@ struct MfmaSplitLayer {
       issue(C);
       wait_tile<2 * N_LOADS>(A);
       compute(A, i);
-    }
-    if (left == 2) {
-      issue(A);
-      wait_tile<2 * N_LOADS>(B);
-      compute(B, i + 1);
+      if (left == 2) {
+        issue(A);
+        wait_tile<2 * N_LOADS>(B);
+        compute(B, i + 1);
+      }
     }
     wait_tile<0>(A);
     wait_tile<0>(B);
@@ -528,11 +572,18 @@ struct MfmaSplitLayer {
     if (lane < 4) cx.tile_lds[3 * PART / 2 + lane] = 0.0f;
     if (fast_end > tb) prefetch_loop<LIK, LAST, GRAD>(cx, mc, tb, fast_end, n, q);
     // ragged tail tile, or unaligned caller buffers: one tile at a time
-    for (int tile = max(tb, fast_end); tile < te; ++tile) {
-      TileIn ti;
-      load_tile_safe(ti, cx, tile * 16, n, q);
-      compute_tile<LIK, LAST, false, GRAD>(ti, cx.tile_lds, cx, mc, tile * 16, n, q);
+    for (int tile = max(tb, fast_end); tile < te; ++tile) tile_alone<LIK, LAST, GRAD, false>(cx, mc, tile, n, q);
+    // (hs is the sum of all rows' loss gradients, dl of their log-likelihoods)
+    if (again_in_fp32(GRAD ? __builtin_isnan(hs) : __builtin_isnan(dl), cx.w_lds, P)) {
+      zero_acc();
+      for (int tile = tb; tile < te; ++tile) tile_alone<LIK, LAST, GRAD, true>(cx, mc, tile, n, q);
     }
+  }
+  template <int LIK, bool LAST, bool GRAD, bool FP32>
+  __device__ __forceinline__ void tile_alone(const StepCtx& cx, const ModelConsts& mc, int tile, int n, int q) {
+    TileIn ti;
+    load_tile_safe(ti, cx, tile * 16, n, q);
+    compute_tile<LIK, LAST, false, GRAD, FP32>(ti, cx.tile_lds, cx, mc, tile * 16, n, q);
   }
 
   // after fold4(x0, y0, x1, y1) row q of lanes holds the sum over the four rows of lanes of x0 (q = 0),

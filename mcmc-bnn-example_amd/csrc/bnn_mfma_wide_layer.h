@@ -175,11 +175,33 @@ struct MfmaWideLayer {
     }
   }
 
+  // GEMM1 of a tile in FP32, the rows read again from memory (rows past the end: the last row); scaled afterwards, since
+  // -2 / ln 2 times a large finite weight may be infinite
+  static __device__ __forceinline__ void gemm1_fp32(const float* s_w, const StepCtx& cx, int row0, int n, int q,
+                                                    f4 (&acc)[NT]) {
+    const float* row = cx.X + (size_t)min(row0 + n, cx.n - 1) * D0;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float b = s_w[oB1 + 16 * t + n];
+      acc[t] = f4{b, b, b, b};
+    }
+#pragma unroll 1
+    for (int k = q; k < D0; k += 4) {
+      const float x = row[k];
+      const float* w = s_w + k * D1 + n;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = mfma_f32(x, w[16 * t], acc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] *= kExp2Scale;
+  }
+
   // GEMM1 + activation + loss gradient + GEMM2 of one tile; `mid` runs before the pointwise stage and `late` in
   // the middle of GEMM2 (the tile loop issues loads there, as registers become free).  PARTS is for
   // the tile-ceiling probe, which times the halves of the instruction mix alone: 1 = the matrix instructions,
   // their operand fetch from LDS and the splits, 2 = the pointwise stage, 3 = the whole tile (what the kernel runs).
-  template <int LIK, bool LAST, bool FULL, int PARTS = 3, class Mid, class Late>
+  // FP32: where a row sum is NaN, GEMM1 in FP32.
+  template <int LIK, bool LAST, bool FULL, int PARTS = 3, bool FP32 = false, class Mid, class Late>
   __device__ __forceinline__ void compute_tile(const RowsA& ra, RowsB& rb, const float* s_w, const __bf16* planes,
                                                const StepCtx& cx, const ModelConsts& mc, int row0, int n, int q,
                                                Mid mid, Late late) {
@@ -230,21 +252,32 @@ struct MfmaWideLayer {
     f2 gx[4][FV];
     if (PARTS & 2) {
       // s = 1 / (1 + 2^t) (kernel_helpers.h:34-42 without the small-|x| identity branch, see prepare_step)
-      float yh[4] = {y_0, y_0, y_0, y_0};
+      float rz;
+      auto row_sums = [&] {
+        float yh[4] = {y_0, y_0, y_0, y_0};
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float w2y = s_w[oW2 + 16 * t + n] * w2_scale;
+        for (int t = 0; t < NT; ++t) {
+          const float w2y = s_w[oW2 + 16 * t + n] * w2_scale;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float e = __builtin_amdgcn_exp2f(acc[t][j]);
-          const float sg = __builtin_amdgcn_rcpf(1.0f + e);
-          acc[t][j] = sg;
-          yh[j] = __builtin_fmaf(w2y, sg, yh[j]);
+          for (int j = 0; j < 4; ++j) {
+            const float e = __builtin_amdgcn_exp2f(acc[t][j]);
+            const float sg = __builtin_amdgcn_rcpf(1.0f + e);
+            acc[t][j] = sg;
+            yh[j] = __builtin_fmaf(w2y, sg, yh[j]);
+          }
+        }
+        rz = row16_reduce4(yh[0], yh[1], yh[2], yh[3]) + __builtin_fmaf(rb.y1, sr2v, rho);
+      };
+      row_sums();
+      if constexpr (FP32) {
+        if (__builtin_amdgcn_ballot_w64(__builtin_isnan(rz)) != 0) {
+          gemm1_fp32(s_w, cx, row0, n, q, acc);
+          row_sums();
         }
       }
       // scaled residual (y - yhat - b2) / scale of the four rows 4 q + j (mcmc_step_ffma.h:293), in bank
       // j of one register; the loss gradient is computed on that one register
-      const float dz = (row16_reduce4(yh[0], yh[1], yh[2], yh[3]) + __builtin_fmaf(rb.y1, sr2v, rho)) * ratio;
+      const float dz = rz * ratio;
       float gz;
       if (LIK == 0) gz = dz * mc.g_scale * __builtin_amdgcn_rcpf(__builtin_fmaf(dz, dz, mc.df));
       else gz = dz * mc.scale_recp;
@@ -351,13 +384,20 @@ struct MfmaWideLayer {
       }
       __builtin_amdgcn_s_setprio(0);
     }
-    for (int tile = max(tb, fast_end); tile < te; ++tile) {
-      RowsA ra;
-      RowsB rb;
-      load_a<false>(ra, cx, tile * 16, n, q);
-      load_b<false>(rb, cx, tile * 16, n, q);
-      compute_tile<LIK, LAST, false>(ra, rb, s_w, planes, cx, mc, tile * 16, n, q, [] {}, [] {});
+    for (int tile = max(tb, fast_end); tile < te; ++tile) tile_alone<LIK, LAST, false>(cx, mc, s_w, planes, tile, n, q);
+    if (again_in_fp32(__builtin_isnan(db2acc), s_w, P)) {  // (the sum of all rows' loss gradients)
+      zero_acc();
+      for (int tile = tb; tile < te; ++tile) tile_alone<LIK, LAST, true>(cx, mc, s_w, planes, tile, n, q);
     }
+  }
+  template <int LIK, bool LAST, bool FP32>
+  __device__ __forceinline__ void tile_alone(const StepCtx& cx, const ModelConsts& mc, const float* s_w,
+                                             const __bf16* planes, int tile, int n, int q) {
+    RowsA ra;
+    RowsB rb;
+    load_a<false>(ra, cx, tile * 16, n, q);
+    load_b<false>(rb, cx, tile * 16, n, q);
+    compute_tile<LIK, LAST, false, 3, FP32>(ra, rb, s_w, planes, cx, mc, tile * 16, n, q, [] {}, [] {});
   }
 
   // The workgroup record in LDS, in columns of four: the dW1 sums in accumulator order (a column is a lane's four

@@ -7,6 +7,10 @@
 
 namespace bnn {
 
+// A number that is infinite, or rounds to an infinite bf16 (beyond 3.3895e38), has no such parts: m and l come out NaN,
+// and so does every product with them.  A wave whose sums come out NaN takes its tiles again, those with a NaN among
+// their row sums on FP32 matrix instructions, which carry infinity as FP32 arithmetic does (again_in_fp32).
+constexpr float LARGEST_BF16 = 0x1.FEp127f;
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
@@ -49,19 +53,24 @@ __device__ __forceinline__ void split2(f2 x, bf2& h, bf2& m, bf2& l) {
   }
 }
 // The parts of w * scale for a weight that stays the same for many rows: the rounding of the product goes into the
-// last part.  An infinite weight becomes a large finite one: parts of infinity would turn every product into NaN,
-// while a weight of 2^120 saturates a hidden unit as infinity does.
+// last part.
 __device__ __forceinline__ void split_scaled(float w, float scale, __bf16& h, __bf16& m, __bf16& l) {
-  float hi = w * scale;
-  float lo = __builtin_fmaf(w, scale, -hi);
-  if (__builtin_fabsf(hi) > 0x1p120f) {
-    hi = __builtin_copysignf(0x1p120f, hi);
-    lo = 0.0f;
-  }
+  const float hi = w * scale;
+  const float lo = __builtin_fmaf(w, scale, -hi);
   h = (__bf16)hi;
   const float r = hi - (float)h;
   m = (__bf16)r;
   l = (__bf16)((r - (float)m) + lo);
+}
+// ... of numbers up to the largest FP32 one: h stays finite
+__device__ __forceinline__ void split2_any(f2 x, bf2& h, bf2& m, bf2& l) {
+  const f2 t = {__builtin_fabsf(x[0]) > LARGEST_BF16 ? __builtin_copysignf(LARGEST_BF16, x[0]) : x[0],
+                __builtin_fabsf(x[1]) > LARGEST_BF16 ? __builtin_copysignf(LARGEST_BF16, x[1]) : x[1]};
+  h = __builtin_convertvector(t, bf2);
+  const f2 r = {x[0] - (float)h[0], x[1] - (float)h[1]};
+  m = __builtin_convertvector(r, bf2);
+  const f2 r2 = {r[0] - (float)m[0], r[1] - (float)m[1]};
+  l = __builtin_convertvector(r2, bf2);
 }
 template <bool DOT = false>
 __device__ __forceinline__ void split4(f4 x, bf4& h, bf4& m, bf4& l) {

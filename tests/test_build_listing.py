@@ -1,5 +1,5 @@
-"""The machine code of the library's own kernels, read from the build: wait states the compiler cannot see are needed,
-because the lane swaps sit in assembly statements."""
+"""The machine code of the library's own kernels, read from the build, where assembly statements hide from the compiler
+what it would otherwise wait for: the matrix instructions in front of lane swaps, and tile loads in flight."""
 import os
 import re
 import subprocess
@@ -58,14 +58,108 @@ def test_the_check_sees_a_swap_behind_a_matrix_instruction():
     assert swaps_too_early(code % "\tv_add_f32_e32 v6, v6, v6\n") == (1, [])  # (the compiler waits for that one)
 
 
-@pytest.mark.parametrize("name", ["bnn_hmc_kernel", "bnn_hmc_kernel_wide"])
-def test_lane_swaps_wait_for_the_matrix_instructions(lib, tmp_path, name):
+LINE = re.compile(r"\s+([a-z]\w+)(?:\s+(.*?))?\s*//\s*([0-9A-Fa-f]+):")
+VREG = re.compile(r"(?<![\w.])v(?:(\d+)|\[(\d+):(\d+)\])(?!\w)")
+VMEM = ("global_", "buffer_", "flat_", "scratch_")
+
+
+def vregs(text):
+    out = set()
+    for one, lo, hi in VREG.findall(text):
+        out.update([int(one)] if one else range(int(lo), int(hi) + 1))
+    return out
+
+
+def functions(listing):
+    name, code = None, []
+    for line in listing.splitlines():
+        if line.endswith(">:"):
+            if code:
+                yield name, code
+            name, code = line.split("<")[1][:-2], []
+        m = LINE.match(line)
+        if m:
+            code.append((m.group(1), m.group(2) or "", int(m.group(3), 16)))
+    if code:
+        yield name, code
+
+
+def used_in_flight(code):
+    """Instructions that use a register a load still in flight will write, over every path through the code.  A load is
+    known to have landed behind a wait for at most k outstanding accesses once k younger ones have been issued (they
+    return in order, so a load may also follow another into the same register)."""
+    at = {a: i for i, (_, _, a) in enumerate(code)}
+    succ = []
+    for i, (op, args, a) in enumerate(code):
+        if op.startswith("s_cbranch") or op == "s_branch":
+            d = int(args.split()[0], 0)
+            target = at[a + 4 + 4 * (d - 65536 if d >= 32768 else d)]
+            succ.append([target] if op == "s_branch" else [i + 1, target])
+        else:
+            assert "setpc" not in op and "swappc" not in op, op
+            succ.append([] if op == "s_endpgm" or i + 1 == len(code) else [i + 1])
+    leaders = {t for i, s in enumerate(succ) if s != [i + 1] for t in s}
+    entry, work, bad = {0: {}}, [0], set()
+    while work:
+        i = work.pop()
+        young = dict(entry[i])  # register -> accesses issued after the load that will write it, at least
+        while True:
+            op, args, a = code[i]
+            if op == "s_waitcnt":
+                m = re.search(r"vmcnt\((\d+)\)", args)
+                if m:
+                    young = {r: y for r, y in young.items() if y < int(m.group(1))}
+            else:
+                load = op.startswith(VMEM) and "load" in op
+                if young and young.keys() & vregs(args.partition(",")[2] if load else args):
+                    bad.add("%x: %s %s" % (a, op, args))
+                if op.startswith(VMEM):
+                    young = {r: y + 1 for r, y in young.items()}
+                    if load:
+                        young.update(dict.fromkeys(vregs(args.partition(",")[0]), 0))
+            if succ[i] != [i + 1] or i + 1 in leaders:
+                break
+            i += 1
+        for t in succ[i]:
+            old = entry.get(t)
+            new = dict(young) if old is None else {r: min(young.get(r, 99), old.get(r, 99)) for r in {*young, *old}}
+            if new != old:
+                entry[t] = new
+                work.append(t)
+    return sorted(bad)
+
+
+def test_the_check_sees_registers_with_a_load_in_flight():
+    def listing(*ops):
+        text = "0000 <k>:\n" + "".join("\t%s  // %X: 0\n" % (op, 4 * i) for i, op in enumerate(ops + ("s_endpgm",)))
+        return next(functions(text))[1]
+
+    two = ("global_load_dwordx4 v[0:3], v9, s[0:1]", "global_load_dword v4, v9, s[0:1]")
+    assert used_in_flight(listing(*two, "s_waitcnt vmcnt(1)", "v_add_f32_e32 v5, v3, v5")) == []
+    assert len(used_in_flight(listing(*two, "s_waitcnt vmcnt(1)", "v_add_f32_e32 v5, v4, v5"))) == 1
+    assert len(used_in_flight(listing(*two, "s_waitcnt vmcnt(1)", "v_mov_b32_e32 v4, 0"))) == 1
+    # the wait is on one of two paths only
+    assert len(used_in_flight(listing(*two, "s_cbranch_scc0 1", "s_waitcnt vmcnt(0)", "v_add_f32_e32 v5, v4, v5"))) == 1
+
+
+def disassemble(tmp_path, name):
     fat, co = str(tmp_path / "fat"), str(tmp_path / "co")
     subprocess.run([os.path.join(LLVM, "llvm-objcopy"), "--dump-section", ".hip_fatbin=" + fat,
                     os.path.join(BUILD, name + ".o"), str(tmp_path / "o")], check=True)
     subprocess.run([os.path.join(LLVM, "clang-offload-bundler"), "--unbundle", "--type=o", "--input=" + fat,
                     "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", "--output=" + co], check=True)
-    listing = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--no-show-raw-insn", co], check=True,
-                             stdout=subprocess.PIPE, text=True).stdout
+    return subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--no-show-raw-insn", co], check=True,
+                          stdout=subprocess.PIPE, text=True).stdout
+
+
+@pytest.mark.parametrize("name", ["bnn_hmc_kernel", "bnn_hmc_kernel_wide"])
+def test_assembly_statements_wait_for_what_they_use(lib, tmp_path, name):
+    listing = disassemble(tmp_path, name)
     swaps, early = swaps_too_early(listing)
     assert swaps > 0 and not early, early[:5]
+    kernels = 0
+    for fn, code in functions(listing):
+        bad = used_in_flight(code)
+        assert not bad, (fn, bad[:5])
+        kernels += 1
+    assert kernels >= 4
