@@ -612,6 +612,7 @@ struct bnnhmc_sampler {
   float* tmp = nullptr;       // evaluation scratch: w | grad | prior (3 * st_stride) ...
   float* tmp_ell = nullptr;   // ... and n_pad rows
   double* tmp_sums = nullptr; // [max_groups][2]
+  double* loss_sums = nullptr;  // LOSS_SUMS doubles: what the forward-only kernel adds up (plans that have it)
   unsigned long long* debug_phase = nullptr;  // set when BNNHMC_DEBUG_PHASE is in the environment
   // Page-locked host memory that kernels read and write (launch_pack): what short calls hand over and return.
   // Several threads may read the chains of one sampler: the mutex is held while a call uses it.
@@ -638,6 +639,10 @@ struct bnnhmc_sampler {
 };
 
 namespace {
+
+// Sums of the forward-only loss kernel at a time, in doubles (512 KB): the samples go through it in batches of
+// LOSS_SUMS / (chunks + 1), 15 of them at least (4096 chunks) and 32768 at most.
+constexpr size_t LOSS_SUMS = 1u << 16;
 
 // size of the staging memory: an evaluation's status, rows, prior terms and gradient
 size_t staging_words(const bnnhmc_sampler* s) {
@@ -1137,6 +1142,7 @@ int bnnhmc_create(const bnnhmc_model* model, const bnnhmc_hmc* hmc, const bnnhmc
       (rc = s->alloc(&s->tmp, (size_t)3 * s->st_stride * eval_groups_max)) ||
       (rc = s->alloc(&s->tmp_ell, (size_t)s->n_pad)) ||
       (rc = s->alloc(&s->tmp_sums, (size_t)2 * eval_groups_max)) ||
+      (s->plan.forward && (rc = s->alloc(&s->loss_sums, LOSS_SUMS))) ||
       (rc = s->alloc(&s->wg_scratch, (size_t)s->plan.resident_wgs * s->plan.wg_scratch_floats)))
     return bail(rc);
   s->workspace = ws;
@@ -1561,8 +1567,8 @@ int bnnhmc_final_loss(bnnhmc_sampler* s, int chain, double* loss1, double* loss2
   if (s->plan.forward) {
     // One workgroup per sample and chunk of rows.  Chunks: enough workgroups to keep the last round of them
     // small (about sixteen rounds in all), but four tiles per wave at least, below which fetching and splitting the
-    // weights takes longer than the rows.  The sums land in the exchange records, which every launch of the
-    // trajectory kernel clears before it uses them.
+    // weights takes longer than the rows.  The sums have a buffer of their own: another thread's evaluation on the same
+    // sampler may run between this kernel and the copy behind it.
     LossArgs a;
     a.n = s->model.n;
     a.n_tiles = (s->model.n + 15) / 16;
@@ -1570,12 +1576,10 @@ int bnnhmc_final_loss(bnnhmc_sampler* s, int chain, double* loss1, double* loss2
     a.X = s->X + (size_t)window * s->model.n * s->model.d0;
     a.y = s->y + (size_t)window * s->n_pad;
     const int waves = 8;
-    const Workspace w = carve_workspace(s->workspace, s->L.P, s->plan.resident_wgs, s->plan.max_groups, s->plan.wide);
-    a.out = (double*)w.partials;
-    const size_t room = (size_t)s->plan.resident_wgs * 2 * w.slot_floats * sizeof(float) / sizeof(double);
+    a.out = s->loss_sums;
     const int wanted = (16 * s->plan.resident_wgs + stored - 1) / stored;
     a.chunks = std::max(1, std::min(wanted, a.n_tiles / (4 * waves)));
-    const int batch = (int)std::min<size_t>((size_t)stored, room / (size_t)(a.chunks + 1));
+    const int batch = (int)std::min<size_t>((size_t)stored, LOSS_SUMS / (size_t)(a.chunks + 1));
     std::vector<double> sums;
     for (int b = 0; b < stored; b += batch) {
       a.n_vectors = std::min(batch, stored - b);
