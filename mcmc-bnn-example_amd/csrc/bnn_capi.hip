@@ -644,9 +644,11 @@ namespace {
 // LOSS_SUMS / (chunks + 1), 15 of them at least (4096 chunks) and 32768 at most.
 constexpr size_t LOSS_SUMS = 1u << 16;
 
-// size of the staging memory: an evaluation's status, rows, prior terms and gradient
+// size of the staging memory: an evaluation's status, rows, prior terms and gradient.  Page-locked memory is scarce:
+// rows beyond 4 MB (where the cost of a copy command no longer counts) are copied instead.
+constexpr int STAGED_ROWS = 1 << 20;
 size_t staging_words(const bnnhmc_sampler* s) {
-  return (size_t)STATUS_READ + s->n_pad + 3 * (size_t)s->st_stride + 8;
+  return (size_t)STATUS_READ + std::min(s->n_pad, STAGED_ROWS) + 3 * (size_t)s->st_stride + 8;
 }
 
 KArgs base_args(const bnnhmc_sampler* s) {
@@ -1533,7 +1535,8 @@ int bnnhmc_eval(bnnhmc_sampler* s, int window, const float* w, float* ell, float
   out.add(s->workspace, STATUS_READ);
   out.add(dp, (int)P);
   out.add(dg, (int)P);
-  out.add(s->tmp_ell, ell ? (int)n : 0);
+  const bool staged = s->model.n <= STAGED_ROWS;
+  out.add(s->tmp_ell, ell && staged ? (int)n : 0);
   out.dst = s->staging;
   HIP_TRY(launch_pack(out, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
@@ -1542,7 +1545,11 @@ int bnnhmc_eval(bnnhmc_sampler* s, int window, const float* w, float* ell, float
   const unsigned* res = s->staging + STATUS_READ;
   if (prior) memcpy(prior, res, P * sizeof(float));
   if (grad) memcpy(grad, res + P, P * sizeof(float));
-  if (ell) memcpy(ell, res + 2 * P, n * sizeof(float));
+  if (ell && staged) memcpy(ell, res + 2 * P, n * sizeof(float));
+  if (ell && !staged) {
+    HIP_TRY(hipMemcpyAsync(ell, s->tmp_ell, n * sizeof(float), hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+  }
   return BNNHMC_OK;
 }
 

@@ -1,5 +1,5 @@
-"""Calls that hand results to the host: final losses of more samples than one batch of sums holds, and several threads
-that read one sampler."""
+"""Calls that hand results to the host: final losses of more samples than one batch of sums holds, several threads that
+read one sampler, rows on either side of the size that goes through page-locked memory."""
 import threading
 
 import numpy as np
@@ -68,4 +68,19 @@ def test_threads_that_read_one_sampler(lib):
     for t in threads:
         t.join()
     assert not wrong, wrong
+    s.close()
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 3, (1 << 20) + 5])
+def test_rows_of_an_evaluation_whatever_their_number(lib, orc, n):
+    model, om = lib.default_model(n=n), ob.Model(22, 40, n, ob.LIK_STUDENT_T, 100.0, 2.2, 200.0)
+    s = lib.create(model, lib.default_hmc(seed=2), lib.default_launch(), 1, 1)
+    th = s.generate_window(0, teacher_scale=0.1, noise_sigma=1.0)
+    w = (0.9 * th).astype(np.float32)
+    X, y = s.get_window_data(0)
+    ell, prior, grad = s.eval(0, w)
+    want = orc.eval_f32(om, X, y, w)
+    np.testing.assert_allclose(ell, want[0], rtol=1e-5, atol=1e-5)
+    assert prior.tobytes() == want[1].tobytes()
+    assert np.abs(grad - want[2]).max() <= 1e-5 * np.abs(want[2]).max()
     s.close()
