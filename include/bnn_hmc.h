@@ -92,7 +92,8 @@ typedef struct bnnhmc_launch {
   int threads;        /* threads per workgroup; default 512 for MFMA (every tile loop), 256 for  */
                       /* FFMA and with wgs_per_cu = 2.  The plain MFMA loop is also built for    */
                       /* 256, 768 and 1024 threads (the last two leave too few registers and    */
-                      /* spill: correct, slower).  64 -> 128 -> 1: 512 (default) or 256           */
+                      /* spill: correct, slower).  64 -> 128 -> 1: 512 (default; spills outside  */
+                      /* its tile loop) or 256                                                   */
   int pipeline;       /* MFMA tile loop: 0 = default: loop 4 at 512 threads, loop 3 otherwise;   */
                       /* 4 = loads issued two tiles ahead with explicit waits, contractions on   */
                       /* v_mfma_f32_16x16x32_bf16 (512 threads only: asking for it with another  */

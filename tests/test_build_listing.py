@@ -163,3 +163,22 @@ def test_assembly_statements_wait_for_what_they_use(lib, tmp_path, name):
         assert not bad, (fn, bad[:5])
         kernels += 1
     assert kernels >= 4
+
+
+def test_tile_loops_of_the_wide_kernel_hardly_touch_scratch(lib, tmp_path):
+    """Full tiles: 192 matrix instructions per trip; two instructions on scratch memory at most where the last step's
+    rows are not written."""
+    seen = []
+    for fn, code in functions(disassemble(tmp_path, "bnn_hmc_kernel_wide")):
+        at = {a: i for i, (_, _, a) in enumerate(code)}
+        trips = []
+        for i, (op, args, a) in enumerate(code):
+            if not (op.startswith("s_cbranch") or op == "s_branch"):
+                continue
+            d = int(args.split()[0], 0)
+            ops = [o for o, _, _ in code[at[a + 4 + 4 * (d - 65536 if d >= 32768 else d)]: i + 1]]
+            if sum("mfma_f32_16x16x32_bf16" in o for o in ops) == 192 and not any("16x16x4_f32" in o for o in ops):
+                trips.append(sum(o.startswith("scratch_") for o in ops))
+        assert trips, fn
+        seen.append(min(trips))
+    assert len(seen) == 4 and max(seen) <= 2, seen
