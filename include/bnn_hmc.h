@@ -198,8 +198,9 @@ int bnnhmc_get_loss_values(const float* loss_values, int n, int n_params, float*
 
 /* ------------------------------------------------------------------------------------------------
  * Sampler level: the phases of mcmc::main_loop (include/mcmc/main.h:117-308) for many windows.
- * Host pointers unless stated.  A sampler is bound to device 0 and one stream; calls on one sampler
- * are not thread-safe, distinct samplers are independent.
+ * Host pointers unless stated.  A sampler is bound to device 0 and one stream.  Calls that only read a
+ * sampler (bnnhmc_get_*, bnnhmc_eval, bnnhmc_final_loss, bnnhmc_window_diagnostics) may come from several threads;
+ * no other call on it may overlap with them or with each other.  Distinct samplers are independent.
  * ---------------------------------------------------------------------------------------------- */
 typedef struct bnnhmc_sampler bnnhmc_sampler;
 

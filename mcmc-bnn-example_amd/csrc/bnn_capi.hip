@@ -615,7 +615,8 @@ struct bnnhmc_sampler {
   double* loss_sums = nullptr;  // LOSS_SUMS doubles: what the forward-only kernel adds up (plans that have it)
   unsigned long long* debug_phase = nullptr;  // set when BNNHMC_DEBUG_PHASE is in the environment
   // Page-locked host memory that kernels read and write (launch_pack): what short calls hand over and return.
-  // Several threads may read the chains of one sampler: the mutex is held while a call uses it.
+  // Calls that only read a sampler may come from several threads: the mutex is held while one of them uses the staging
+  // memory or the evaluation buffers above.
   unsigned* staging = nullptr;
   std::mutex staging_mutex;
   // timing
@@ -1561,6 +1562,7 @@ int bnnhmc_final_loss(bnnhmc_sampler* s, int chain, double* loss1, double* loss2
       std::max(0, std::min(s->hmc.n_samples, s->transitions_done - s->hmc.burn_in));
   if (stored == 0) return fail(BNNHMC_ERR_STATE, "chain %d has no kept samples yet", chain);
   const int window = chain / s->cpw;
+  std::lock_guard<std::mutex> lock(s->staging_mutex);
   const float* base = s->samples + (size_t)chain * s->hmc.n_samples * s->L.P;
   double l1 = 0, l2 = 0, fl = 0;
   int step = 0;
@@ -1574,8 +1576,8 @@ int bnnhmc_final_loss(bnnhmc_sampler* s, int chain, double* loss1, double* loss2
   if (s->plan.forward) {
     // One workgroup per sample and chunk of rows.  Chunks: enough workgroups to keep the last round of them
     // small (about sixteen rounds in all), but four tiles per wave at least, below which fetching and splitting the
-    // weights takes longer than the rows.  The sums have a buffer of their own: another thread's evaluation on the same
-    // sampler may run between this kernel and the copy behind it.
+    // weights takes longer than the rows.  The sums have a buffer of their own: nothing else on the sampler's stream touches
+    // them between this kernel and the copy behind it.
     LossArgs a;
     a.n = s->model.n;
     a.n_tiles = (s->model.n + 15) / 16;

@@ -37,9 +37,11 @@ def test_final_loss_of_more_samples_than_one_batch(lib, orc):
     s.close()
 
 
-def test_threads_that_read_one_sampler(lib):
+@pytest.mark.parametrize("losses_by", ["forward kernel", "whole evaluations"])
+def test_threads_that_read_one_sampler(pkg, lib, losses_by):
     n, keep, chains = 2000, 6, 8
-    s = sampler(lib, n, keep, L=3, windows=2, chains=4)
+    layer = {"forward kernel": pkg.LAYER_MFMA, "whole evaluations": pkg.LAYER_FFMA}[losses_by]
+    s = sampler(lib, n, keep, L=3, windows=2, chains=4, launch=lib.default_launch(layer=layer))
     rng = np.random.default_rng(0)
     ws = [(s.get_samples(0)[0] + rng.normal(0, 0.01, s.P)).astype(np.float32) for _ in range(chains)]
 
@@ -49,7 +51,7 @@ def test_threads_that_read_one_sampler(lib):
         return (s.get_samples(c).tobytes(), state["w"].tobytes(), state["grad"].tobytes(), state["eps"],
                 state["n_accepted"], ell.tobytes(), prior.tobytes(), grad.tobytes())
 
-    want, losses = [read(c) for c in range(chains)], s.final_loss(3)
+    want, losses = [read(c) for c in range(chains)], {c: s.final_loss(c) for c in (3, 5)}
     wrong = []
 
     def work(c):
@@ -57,12 +59,13 @@ def test_threads_that_read_one_sampler(lib):
             if read(c) != want[c]:
                 wrong.append(c)
 
-    def work_losses():
+    def work_losses(c):
         for _ in range(40):
-            if s.final_loss(3) != losses:
+            if s.final_loss(c) != losses[c]:
                 wrong.append("losses")
 
-    threads = [threading.Thread(target=work, args=(c,)) for c in range(chains)] + [threading.Thread(target=work_losses)]
+    threads = [threading.Thread(target=work, args=(c,)) for c in range(chains)]
+    threads += [threading.Thread(target=work_losses, args=(c,)) for c in losses]
     for t in threads:
         t.start()
     for t in threads:
