@@ -82,7 +82,8 @@ typedef struct bnnhmc_launch {
                       /* batches, transitions_per_launch transitions at a time, and what does not  */
                       /* fill a batch runs in smaller, wider ones.  64 -> 128 -> 1: 4, a smaller    */
                       /* last batch widened.  Step operator: 256.  On few rows all of these are      */
-                      /* narrower: about one 16-row tile per SIMD (64 -> 128 -> 1: per wave).        */
+                      /* narrower: about one 16-row tile per SIMD (64 -> 128 -> 1: per wave, but 4   */
+                      /* at least in the sampler).                                                 */
                       /* Results are bit-reproducible for                                          */
                       /* a fixed count; with 0 and more chains than fit at once, which launches run */
                       /* wider depends on how a job is cut into bnnhmc_run calls and on that time   */

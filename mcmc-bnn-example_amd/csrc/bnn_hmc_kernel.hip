@@ -873,7 +873,7 @@ const void* hmc_kernel_for(int d0, int d1, int layer, int lik, int threads, int 
   using MH = MfmaSplitLayer<22, 40>;
   using F = FfmaLayer<22, 40>;
   if (layer == 0 && pipeline == 4) {
-    // hidden units 32 .. 39 on 4x4 blocks (bnn_mfma_split_layer.h): prefetched loop, 512 threads only
+    // contractions on bf16 parts (bnn_mfma_split_layer.h): prefetched loop, 512 threads only
     if (threads == 512) return lik == 0 ? kernel_ptr<MH, 0, 512>() : kernel_ptr<MH, 1, 512>();
   } else if (layer == 0 && pipeline == 2) {
     // The prefetched loop is built for 512 threads only.  Its loads are issued from inline assembly

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(T) void hmc_kernel_wide(const KArgs a) {
   // the last four hold a double): the gradient is dead once the leapfrog update has used it
   float* s_g = s_m + P_AL;
   float* s_red = s_g;
-  __bf16* s_planes = reinterpret_cast<__bf16*>(s_red + SLOT);  // W1 of this step, split (Layer::store_split)
+  __bf16* s_planes = reinterpret_cast<__bf16*>(s_red + SLOT);  // W1 of this step, split (Layer::store_split8)
   __shared__ double s_wsum[W];
   __shared__ unsigned long long s_hash[W];
   __shared__ int s_flag;
@@ -235,8 +235,9 @@ __global__ __launch_bounds__(T) void hmc_kernel_wide(const KArgs a) {
         //      columns over all G records: thread (record lane rl = tid / CS, column c = tid % CS) adds records rl,
         //      rl + T / CS, ... in order, the record lanes of a wave are added by a fixed xor tree and the others in
         //      order through LDS.  Phase 2, once every slice is stored: everyone reads the totals.  CS is such that a
-        //      thread has eight records at most, all in flight at once; a workgroup then has one slice or none, and
-        //      nobody waits for a second trip to memory. ----
+        //      thread has eight records at most, all in flight at once, and a workgroup one slice or none where G is a
+        //      power of two, so that nobody waits for a second trip to memory.  (Other groups, and 256
+        //      threads: a few workgroups may have a second slice; 256 threads at G = 256: 16 records, CS is 16 at least.) ----
         constexpr int NCOL = P_AL / 4;
         float* tot = a.totals + (size_t)group * SLOT;
         f4* s_x = reinterpret_cast<f4*>(s_red);    // free: this step's record has been published

@@ -505,11 +505,7 @@ struct MfmaSplitLayer {
     const int back = __builtin_amdgcn_readfirstlane(cx.back);
     const int back_next = __builtin_amdgcn_readfirstlane(cx.back_next);
     const int len = te - tb;
-    int nk = 2, nback = back;
-    while (nk >= len) {  // (a run of one tile is the same tile in either direction)
-      nk -= len;
-      nback = back_next;
-    }
+    int nk = 2, nback = back;  // (len > KEPT)
     auto issue = [&](TileRaw& r) {
       issue_tile(r, cx, lp, __builtin_amdgcn_readfirstlane(walk(tb, te, nk, nback)));
       if (++nk == len) {

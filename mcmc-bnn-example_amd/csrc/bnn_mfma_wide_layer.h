@@ -24,8 +24,8 @@ namespace bnn {
 // Why split: v_mfma_f32_16x16x4_f32 runs at 64 flop per cycle and SIMD and shares its pipe with the vector
 // instructions; the bf16 form runs at 1024 on a pipe of its own.  x = h + m + l with three bf16 parts is exact
 // for a 24-bit significand, and the six products hh, hm, mh, hl, lh, mm leave out ml, lm and ll, of random sign and
-// 2^-27 of a product each on average (2^-24 at most): less than the FP32 rounding of one addition, of which there is
-// one per 32 products instead of one per 4.  So the contraction costs 6/16 of the FP32 time, off the vector pipe, at
+// 2^-27 of a product each on average (2^-24 at most): less than the FP32 rounding of one addition, of which GEMM1 has
+// 12 per 64 products (six of the parts per 32) instead of 16, GEMM2 three per tile instead of four.  So the contraction costs 6/16 of the FP32 time, off the vector pipe, at
 // FP32 precision (measured against 64 bits: as close or closer).  A tile took 4.46 us per SIMD, now 2.5; what limits
 // it is power (the shader clock drops from 2.39 to 2.1 GHz).
 // GEMM2 has only 16 rows to contract per tile and 32 k slots per instruction: two products share an

@@ -95,7 +95,7 @@ def test_eval_matches_oracle(pkg, lib, orc, layer, kind, n, G):
 def test_alternative_tile_loops_match_oracle(pkg, lib, orc, pipeline, threads, kind):
     """The software-pipelined (1), prefetched (2: three 16-wide hidden tiles) and plain (3) tile loops and
     other workgroup sizes stay selectable through the launch parameters; they must give the same gradients as
-    the default loop (4: hidden units 32 .. 39 on 4x4 blocks), here asked for by name.  4101 rows: 256 full
+    the default loop (4: contractions on bf16 parts), here asked for by name.  4101 rows: 256 full
     tiles and a ragged one."""
     say("tile loop %d, %d threads, %s" % (pipeline, threads, kind))
     n = 4101
