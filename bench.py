@@ -235,7 +235,8 @@ def main():
     split = wide or (args.layer == "mfma" and args.pipeline in (0, 4) and args.threads in (0, 512) and wgs_per_cu == 1)
     peak = PEAK_SPLIT_TFLOPS if split else PEAK_TFLOPS
     kernel_key = "hmc_kernel_wide_64x128" if wide else "hmc_kernel_%s_22x40" % args.layer
-    bytes_per_eval = measured_traffic(kernel_key)
+    # (measured on the default tile loop of each network, and on the FFMA layer)
+    bytes_per_eval = measured_traffic(kernel_key) if split or args.layer == "ffma" else None
 
     out = {
         "metric": "leapfrog grad-evals/sec (minutes for 200 windows x 800 samples derived), 1 MI355X",
