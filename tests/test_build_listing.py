@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+import __graft_entry__
+
 BUILD = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mcmc-bnn-example_amd", "build")
 LLVM = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
 # wait states between a matrix instruction of up to eight passes (16x16x32 bf16, 16x16x4 and 4x4x1 f32) and a vector
@@ -143,6 +145,8 @@ def test_the_check_sees_registers_with_a_load_in_flight():
 
 
 def disassemble(tmp_path, name):
+    if not os.path.exists(os.path.join(BUILD, name + ".o")):
+        __graft_entry__.build()
     fat, co = str(tmp_path / "fat"), str(tmp_path / "co")
     subprocess.run([os.path.join(LLVM, "llvm-objcopy"), "--dump-section", ".hip_fatbin=" + fat,
                     os.path.join(BUILD, name + ".o"), str(tmp_path / "o")], check=True)

@@ -29,12 +29,13 @@ def check(got, want, what, rel=1e-5):
 
 
 # n = 1000 at one workgroup: runs of 7 and 8 tiles; 100 at one: one tile per wave; at the default: every wave one tile
-@pytest.mark.parametrize("d0,d1", [(22, 40), (64, 128)])
-@pytest.mark.parametrize("n,G", [(5, 1), (100, 1), (1000, 1), (1000, 0), (4099, 3)])
-def test_features_without_parts(lib, orc, d0, d1, n, G):
+@pytest.mark.parametrize("d0,d1,n,G,threads", [(d0, d1, n, G, 0) for d0, d1 in [(22, 40), (64, 128)] for n, G in
+                                               [(5, 1), (100, 1), (1000, 1), (1000, 0), (4099, 3)]] +
+                         [(64, 128, 500, 1, 256)])
+def test_features_without_parts(lib, orc, d0, d1, n, G, threads):
     model, om = student(lib, n, d0, d1)
     X, y, w = window(orc, d0, d1, n)
-    s = lib.create(model, lib.default_hmc(seed=3), lib.default_launch(cus_per_chain=G), 1, 1)
+    s = lib.create(model, lib.default_hmc(seed=3), lib.default_launch(cus_per_chain=G, threads=threads), 1, 1)
     plain = orc.eval_f32(om, X, y, w)
     for value in (np.inf, -np.inf, HUGE, -HUGE):
         Xv = X.copy()
